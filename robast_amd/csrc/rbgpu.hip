@@ -1800,7 +1800,6 @@ int rbgpu_trace(rb_ctx* ctx, const rb_scene* scene, const rb_trace_opts* opts, r
             HIPCHK(ctx, hipEventSynchronize(ctx->stage_ev[part++]));
           else
             HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-  dev.settled = true;
         }
         const size_t m = std::min(arrays[k].bytes - done, have - (begin + done));
         memcpy(static_cast<char*>(arrays[k].host) + done, pinned + begin + done, m);
@@ -1813,6 +1812,7 @@ int rbgpu_trace(rb_ctx* ctx, const rb_scene* scene, const rb_trace_opts* opts, r
         HIPCHK(ctx, hipMemcpyAsync(arrays[k].host, at[k], arrays[k].bytes, hipMemcpyDeviceToHost, ctx->stream));
   }
   HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+  dev.settled = true;
   float ms = 0, kms = 0;
   HIPCHK(ctx, hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
   HIPCHK(ctx, hipEventElapsedTime(&kms, ctx->evk0, ctx->evk1));
