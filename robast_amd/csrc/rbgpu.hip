@@ -1732,7 +1732,7 @@ int rbgpu_trace(rb_ctx* ctx, const rb_scene* scene, const rb_trace_opts* opts, r
     if (rays->last_node) arrays[count++] = {rays->last_node, ni, true};
     if (cap > 0) arrays[count++] = {rays->path_node, ni * size_t(cap), true};
     for (int k = 0; k < count; k++) total += arrays[k].bytes;
-    dev.reserve(total);
+    dev.reserve(DevRays::room<char>(int64_t(total)));
     HIPCHK(ctx, dev.alloc(&base, int64_t(total)));
     if (total <= kStageBytes && dev.mine) pinned = stage_of(ctx, total);
     size_t off = 0, sent = 0;

@@ -2,7 +2,8 @@
 // memory, for tests of its host code without a GPU. Copies are queued and run
 // when the stream or an event after them is waited for; kernels do nothing.
 // fake_fail makes one wait fail (its copies stay queued); fake_pending counts
-// the copies still queued, fake_stream_waits the waits for the stream.
+// the copies still queued, fake_stream_waits the waits for the stream,
+// fake_mallocs the allocations of device memory.
 #include <cstdlib>
 #include <cstring>
 #include <deque>
@@ -15,7 +16,7 @@ struct Copy {
 };
 std::deque<Copy> queue;
 long done = 0;  // copies run so far
-int fail_stream = 0, fail_event = 0, stream_waits = 0;
+int fail_stream = 0, fail_event = 0, stream_waits = 0, mallocs = 0;
 struct Event {
   long after;
 };
@@ -34,10 +35,11 @@ extern "C" {
 void fake_fail(int event, int stream) {
   fail_event = event;
   fail_stream = stream;
-  stream_waits = 0;
+  stream_waits = mallocs = 0;
 }
 long fake_pending() { return long(queue.size()); }
 int fake_stream_waits() { return stream_waits; }
+int fake_mallocs() { return mallocs; }
 
 void** __hipRegisterFatBinary(const void*) {
   static void* h;
@@ -68,7 +70,7 @@ int hipGetSymbolAddress(void** p, const void*) {
   static char symbol;
   return *p = &symbol, 0;
 }
-int hipMalloc(void** p, size_t n) { return *p = std::calloc(n, 1), 0; }
+int hipMalloc(void** p, size_t n) { return mallocs++, *p = std::calloc(n, 1), 0; }
 int hipFree(void* p) { return run_to(all()), std::free(p), 0; }
 int hipHostMalloc(void** p, size_t n, unsigned) { return *p = std::calloc(n, 1), 0; }
 int hipHostFree(void* p) { return hipFree(p); }

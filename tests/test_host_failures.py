@@ -31,9 +31,9 @@ for ev, st in ((event, stream), (0, 0)):
     fake.fake_fail(ev, st)
     try:
         ctx.trace(scene, make_rays(soa), n, mgr.trace_opts(order=1))
-        print("ok", fake.fake_pending(), fake.fake_stream_waits())
+        print("ok", fake.fake_pending(), fake.fake_stream_waits(), fake.fake_mallocs())
     except RbError:
-        print("failed", fake.fake_pending(), fake.fake_stream_waits())
+        print("failed", fake.fake_pending(), fake.fake_stream_waits(), fake.fake_mallocs())
 assert all((soa[f] == want[f]).all() for f in soa)
 """
 
@@ -68,5 +68,13 @@ def test_no_copy_outlives_a_failed_call(host_runtime, n, event, stream):
 @pytest.mark.parametrize("n, waits", [(1, 2), (149952, 2), (250000, 1)])
 def test_a_call_waits_no_more_than_it_has_to(host_runtime, n, waits):
     """Staged: for the last part and for the timing events; array by array: once."""
-    for state, pending, waited in _run(host_runtime, n, 0, 0):
+    for state, pending, waited, _ in _run(host_runtime, n, 0, 0):
         assert (state, pending, int(waited)) == ("ok", "0", waits)
+
+
+# ray arrays of whole and of broken steps of the work area's 256 bytes, staged
+# or not
+@pytest.mark.parametrize("n", [1, 64, 1000, 149952, 150001, 250001])
+def test_a_second_call_allocates_nothing(host_runtime, n):
+    first, second = _run(host_runtime, n, 0, 0)
+    assert first[3] == "1" and second[3] == "0"
