@@ -286,11 +286,14 @@ template <bool WAVE> __device__ __forceinline__ void stage_lane(const DScene& S)
 // it only to record a path): read from the kernel's arguments when asked for.
 // Thirteen pointers kept through the loop would cost it their scalar
 // registers, which spill.
+// (`args` comes from the kernel's body: in a function that is not inlined
+// into it, the builtin gives null.)
 template <typename ARGS> struct KernelRays {
+  typedef const RB_UNIFORM_AS char* Bytes;
   int32_t path_cap;
+  const char* args;
   __device__ __forceinline__ RayIO rays() const {
-    typedef const RB_UNIFORM_AS char* Bytes;
-    Bytes k = (Bytes)__builtin_amdgcn_kernarg_segment_ptr();
+    Bytes k = (Bytes)uniform(args);
     asm volatile("" : "+s"(k));  // (read here, not where the kernel began)
     const RB_UNIFORM_AS RayIO* a = (const RB_UNIFORM_AS RayIO*)(k + offsetof(ARGS, io));
     RayIO r;
@@ -681,7 +684,8 @@ __global__ void __launch_bounds__(kTraceBlock) RB_WAVE_ATTR(WAVE)
   L.cand = {cand_node + threadIdx.x, cand_tn + threadIdx.x};
   L.ray = P.id_base + uint64_t(i);
   NoRecord rec;
-  const KernelRays<TraceArgs<DSceneOf<MAXD, BORDERS, (MAXD > 1), false, LENS, SOLVER, WAVE>>> io{A.io.path_cap};
+  const KernelRays<TraceArgs<DSceneOf<MAXD, BORDERS, (MAXD > 1), false, LENS, SOLVER, WAVE>>> io{
+      A.io.path_cap, (const char*)__builtin_amdgcn_kernarg_segment_ptr()};
   trace_lane<MIXED>(S, P, io, i, L, rec, act, &i);
   if (!act) return;
   if (rr)
