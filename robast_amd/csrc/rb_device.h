@@ -92,6 +92,10 @@ struct DScene {
   int32_t stage_lo, stage_n;
   // likewise the first leaf_stage_n leaves, the top node's (at most kLeafStage)
   int32_t leaf_stage_n;
+  // many placed shapes have one structure (type; for composites operation and
+  // operands' structures), such as the facets of a mirror measured one by one:
+  // see each_shape
+  bool families;
   // deepest boolean nesting the navigation code is compiled for, and
   // whether it handles border-surface conditions (roughness, Lambertian)
   static constexpr int max_depth = kMaxCsgDepth;
@@ -119,14 +123,19 @@ constexpr int kLeafStage = 128; // 4 KB
 // roots); the lane kernels for scenes with neither (and no ALens) are
 // compiled without it (160 bytes against 288, no VGPR spills).
 // WAVE: the kernels that navigate a wavefront at a time (rb_wave.h).
+// FAM: lanes with a shape each (each_shape) are compiled in. In the one-level
+// lane kernels that costs the other scenes nothing; the work-queue and the
+// deep kernels have a form of their own for scenes with families (the extra
+// calls cost theirs: light guides 1e6 rays 1 %, a lens 3, deep mixed 8).
 template <int MAXD, bool BORDERS = false, bool EXT = (MAXD > 1), bool BOX = false, bool LENS = true,
-          bool SOLVER = true, bool WAVE = false>
+          bool SOLVER = true, bool WAVE = false, bool FAM = (MAXD == 1 && !BOX)>
 struct DSceneOf : DScene {
   static constexpr int max_depth = MAXD;
   static constexpr bool borders_on = BORDERS;
   static constexpr bool ext_on = EXT;
   static constexpr bool box_on = BOX;
   static constexpr bool wave_on = WAVE;
+  static constexpr bool families_on = FAM;
   static constexpr bool lens_on = LENS;
   static constexpr unsigned shape_set = (EXT ? kShapesExt : 0u) | (SOLVER ? kShapesSolver : 0u);
 };
@@ -168,16 +177,16 @@ struct ShapeView {
   const DShape* shapes;
   const double* params;
 };
-// One shape of a view, read with scalar loads: the caller's active lanes all
-// ask for the same shape.
-struct ShapeRef {
+// One shape of a view. ONE: the caller's active lanes all ask for the same
+// shape, which is read with scalar loads; otherwise each lane reads its own.
+template <bool ONE = true> struct ShapeRef {
   ShapeView V;
   ShapePtr sh;
   ParamPtr p;
   int type;
   __device__ __forceinline__ ShapeRef(const ShapeView& view, int shape)
       : V{uniform(view.shapes), uniform(view.params)} {
-    sh = (ShapePtr)V.shapes + uniform(shape);
+    sh = (ShapePtr)V.shapes + (ONE ? uniform(shape) : shape);
     p = (ParamPtr)V.params + sh->off;
     type = sh->type;
   }
@@ -188,23 +197,40 @@ struct ShapeRef {
     return (ParamPtr)V.params + ((ShapePtr)V.shapes + child(side))->box;
   }
 };
-// Runs f(u) once for each distinct shape u among the active lanes, every lane
-// in its own shape's turn: inside, the shape is uniform. The lanes of a
-// coherent wavefront, and all placements of one volume, share their shape, so
-// there are rarely more than two or three turns. (The loop runs over a lane
+// Runs f(u) once for each distinct value u among the active lanes, every lane
+// in its own value's turn: inside, u is uniform. (The loop runs over a lane
 // mask: its condition is uniform, so no lane leaves before its wavefront and
 // f stays inside the loop.)
-template <typename F> __device__ __forceinline__ void each_shape(int shape, F&& f) {
+template <typename F> __device__ __forceinline__ void in_turns(int value, F&& f) {
 #ifndef RB_HOST_EMULATION
   for (unsigned long long left = __ballot(1); left != 0ull;) {
-    const int u = __builtin_amdgcn_readlane(shape, __ffsll(left) - 1);
-    const bool mine = shape == u;
+    const int u = __builtin_amdgcn_readlane(value, __ffsll(left) - 1);
+    const bool mine = value == u;
     left &= ~__ballot(mine);
     if (mine) f(u);
   }
 #else
-  f(shape);
+  f(value);
 #endif
+}
+// Runs f(one, u) for each lane's shape u: in turns, every lane in its own
+// shape's (one = true, u uniform: the shape's data come by scalar loads), or,
+// in scenes with `families`, where the lanes name more than one shape, once for
+// all lanes, each reading its own shape with vector loads (one = false). The
+// lanes of a coherent wavefront, and all placements of one volume, share their
+// shape, so elsewhere there are rarely more than two or three turns, and they
+// are cheaper (in turns and together, us: two-level facets 2e5 rays 480 and
+// 588, aspheric mirrors 1.9e5 555 and 628, a lens 1e6 1199 and 1274). But rays
+// in random order on 85 facets with a shape each name 45 (1e5 rays 1240 and
+// 171; gradient of 8 x 3e4 rays 2250 and 370).
+template <typename F> __device__ __forceinline__ void each_shape(bool families, int shape, F&& f) {
+#ifndef RB_HOST_EMULATION
+  if (families && __ballot(shape != __builtin_amdgcn_readfirstlane(shape)) != 0ull) {
+    f(std::false_type(), shape);
+    return;
+  }
+#endif
+  in_turns(shape, [&](int u) { f(std::true_type(), u); });
 }
 
 template <typename T>
@@ -1630,17 +1656,19 @@ __device__ __forceinline__ bool sbox_ray(ParamPtr b, V3<T> q, V3<T> d) {
   return t0 <= t1 * T(1.0001) + T(1e-3);
 }
 
-// Shape queries, one shape for all active lanes (each_shape).
-template <typename T, int D, unsigned SH, bool BOX = false> struct Csg {
-  using Sub = Csg<T, D - 1, SH, BOX>;
+// Shape queries, one shape for all active lanes or (ONE = false) one per lane
+// (each_shape).
+template <typename T, int D, unsigned SH, bool BOX = false, bool ONE = true> struct Csg {
+  using Sub = Csg<T, D - 1, SH, BOX, ONE>;
+  using Ref = ShapeRef<ONE>;
   // child `side` (0 left, 1 right) contains q: outside its box it does not
-  __device__ __forceinline__ static bool child_in(const ShapeRef& R, int side, V3<T> q) {
+  __device__ __forceinline__ static bool child_in(const Ref& R, int side, V3<T> q) {
     const ParamPtr m = R.placement(side);
     const V3<T> lq = m2l<T>(m, m + 9, q);
     return (!BOX || sbox_has<T>(R.child_box(side), lq)) && Sub::contains(R.V, R.child(side), lq);
   }
   __device__ RB_CSG_FN static bool contains(ShapeView V, int shape, V3<T> q) {
-    const ShapeRef R(V, shape);
+    const Ref R(V, shape);
     if (R.type != RB_SHAPE_COMPOSITE) return prim_contains<T, SH>(R.type, R.p, q);
     const int op = R.sh->op;
     bool a = child_in(R, 0, q);
@@ -1650,7 +1678,7 @@ template <typename T, int D, unsigned SH, bool BOX = false> struct Csg {
   }
   // distance to child `side`; an entry (out) along a ray that misses the
   // child's box is kBig without evaluating the child
-  __device__ static Hit child(const ShapeRef& R, int side, bool out, V3<T> q, V3<T> d) {
+  __device__ static Hit child(const Ref& R, int side, bool out, V3<T> q, V3<T> d) {
     const ParamPtr m = R.placement(side);
     const int c = R.child(side);
     V3<T> lq = m2l<T>(m, m + 9, q), ld = m2lv<T>(m, d);
@@ -1664,7 +1692,7 @@ template <typename T, int D, unsigned SH, bool BOX = false> struct Csg {
   // soon as the iteration has passed it; the accumulated distance only grows,
   // so this changes no accepted result.
   __device__ RB_CSG_FN static Hit dist_out(ShapeView V, int shape, V3<T> q, V3<T> d, double lim = kBig) {
-    const ShapeRef R(V, shape);
+    const Ref R(V, shape);
     if (R.type != RB_SHAPE_COMPOSITE) return {double(prim_dist_out<T, SH>(R.type, R.p, q, d)), 0u, 0u};
     const int op = R.sh->op;
     if (op == RB_OP_UNION) {
@@ -1712,7 +1740,7 @@ template <typename T, int D, unsigned SH, bool BOX = false> struct Csg {
     return {kBig, 0u, 0u};
   }
   __device__ RB_CSG_FN static Hit dist_in(ShapeView V, int shape, V3<T> q, V3<T> d) {
-    const ShapeRef R(V, shape);
+    const Ref R(V, shape);
     if (R.type != RB_SHAPE_COMPOSITE) return {double(prim_dist_in<T, SH>(R.type, R.p, q, d)), 0u, 1u};
     const int op = R.sh->op;
     if (op != RB_OP_UNION) {  // leave A, or for a difference enter B, for an intersection leave B
@@ -1741,7 +1769,7 @@ template <typename T, int D, unsigned SH, bool BOX = false> struct Csg {
   // normal of the leaf surface `path` (bits consumed from bit 0); the lanes
   // may name different leaves of the shape
   __device__ RB_CSG_FN static V3<T> normal(ShapeView V, int shape, uint32_t path, int depth, V3<T> q, V3<T> d) {
-    const ShapeRef R(V, shape);
+    const Ref R(V, shape);
     if (R.type != RB_SHAPE_COMPOSITE) return prim_normal<T, SH>(R.type, R.p, q, d);
     const int side = depth > 0 ? int(path & 1u) : 0;
     V3<T> out = mk<T>(T(0), T(0), T(1));
@@ -1759,7 +1787,7 @@ template <typename T, int D, unsigned SH, bool BOX = false> struct Csg {
   // off by `back` (the mixed form's root polish). Returns kBig on failure.
   __device__ RB_CSG_FN static double polish(ShapeView V, int shape, uint32_t path, int depth, bool exiting, V3<T> q,
                                   V3<T> d, T s0, T back) {
-    const ShapeRef R(V, shape);
+    const Ref R(V, shape);
     if (R.type != RB_SHAPE_COMPOSITE) {
       T t0 = s0 - back > T(0) ? s0 - back : T(0);
       V3<T> q0 = axpy(q, t0, d);
@@ -1779,26 +1807,27 @@ template <typename T, int D, unsigned SH, bool BOX = false> struct Csg {
   }
 };
 // depth exhausted: primitives only (the host rejects deeper expressions)
-template <typename T, unsigned SH, bool BOX> struct Csg<T, 0, SH, BOX> {
+template <typename T, unsigned SH, bool BOX, bool ONE> struct Csg<T, 0, SH, BOX, ONE> {
+  using Ref = ShapeRef<ONE>;
   __device__ RB_CSG0_FN static bool contains(ShapeView V, int shape, V3<T> q) {
-    const ShapeRef R(V, shape);
+    const Ref R(V, shape);
     return prim_contains<T, SH>(R.type, R.p, q);
   }
   __device__ RB_CSG0_FN static Hit dist_out(ShapeView V, int shape, V3<T> q, V3<T> d, double = kBig) {
-    const ShapeRef R(V, shape);
+    const Ref R(V, shape);
     return {double(prim_dist_out<T, SH>(R.type, R.p, q, d)), 0u, 0u};
   }
   __device__ RB_CSG0_FN static Hit dist_in(ShapeView V, int shape, V3<T> q, V3<T> d) {
-    const ShapeRef R(V, shape);
+    const Ref R(V, shape);
     return {double(prim_dist_in<T, SH>(R.type, R.p, q, d)), 0u, 1u};
   }
   __device__ RB_CSG0_FN static V3<T> normal(ShapeView V, int shape, uint32_t, int, V3<T> q, V3<T> d) {
-    const ShapeRef R(V, shape);
+    const Ref R(V, shape);
     return prim_normal<T, SH>(R.type, R.p, q, d);
   }
   __device__ RB_CSG0_FN static double polish(ShapeView V, int shape, uint32_t, int, bool exiting, V3<T> q, V3<T> d, T s0,
                                   T back) {
-    const ShapeRef R(V, shape);
+    const Ref R(V, shape);
     T t0 = s0 - back > T(0) ? s0 - back : T(0);
     V3<T> q0 = axpy(q, t0, d);
     T t = exiting ? prim_dist_in<T, SH>(R.type, R.p, q0, d) : prim_dist_out<T, SH>(R.type, R.p, q0, d);
@@ -1809,7 +1838,13 @@ template <typename T, unsigned SH, bool BOX> struct Csg<T, 0, SH, BOX> {
 // Runs f(std::integral_constant<int, D>) for the nesting depth of shape u, so
 // that a primitive or a single boolean level does not pay for the deepest
 // unrolled form. Scenes typed DSceneOf<1> compile no deeper form at all.
-template <typename SC, typename F> __device__ __forceinline__ void by_depth(const SC& S, int u, F&& f) {
+// (Lanes with a shape each, one = false, all take the scene's deepest form.)
+template <typename SC, typename ONE, typename F>
+__device__ __forceinline__ void by_depth(const SC& S, int u, ONE one, F&& f) {
+  if constexpr (!one()) {
+    f(std::integral_constant<int, SC::max_depth>());
+    return;
+  }
   switch (((ShapePtr)S.shapes + u)->depth) {
     case 0: f(std::integral_constant<int, 0>()); break;
     case 1: f(std::integral_constant<int, 1>()); break;
@@ -1824,31 +1859,33 @@ template <typename SC, typename F> __device__ __forceinline__ void by_depth(cons
 }
 template <typename SC> __device__ __forceinline__ ShapeView shape_view(const SC& S) { return {S.shapes, S.params}; }
 
-// Entry points: each lane's own shape, in turns.
+// Entry points: each lane's own shape.
 template <typename T, typename SC>
 __device__ __forceinline__ V3<T> shape_normal(const SC& S, int shape, uint32_t leaf, V3<T> q, V3<T> d) {
   const uint32_t path = leaf & 0xffffffu;
   const int depth = int(leaf >> 24);
   V3<T> n;
-  each_shape(shape, [&](int u) {
-    by_depth(S, u, [&](auto D) { n = Csg<T, D(), SC::shape_set, SC::box_on>::normal(shape_view(S), u, path, depth, q, d); });
+  each_shape(SC::families_on && S.families, shape, [&](auto one, int u) {
+    by_depth(S, u, one, [&](auto D) {
+      n = Csg<T, D(), SC::shape_set, SC::box_on, one()>::normal(shape_view(S), u, path, depth, q, d);
+    });
   });
   return n;
 }
 template <typename T, typename SC>
 __device__ __forceinline__ bool shape_contains(const SC& S, int shape, V3<T> q) {
   bool in;
-  each_shape(shape, [&](int u) {
-    by_depth(S, u, [&](auto D) { in = Csg<T, D(), SC::shape_set, SC::box_on>::contains(shape_view(S), u, q); });
+  each_shape(SC::families_on && S.families, shape, [&](auto one, int u) {
+    by_depth(S, u, one, [&](auto D) { in = Csg<T, D(), SC::shape_set, SC::box_on, one()>::contains(shape_view(S), u, q); });
   });
   return in;
 }
 template <typename T, typename SC>
 __device__ __forceinline__ Hit shape_dist(const SC& S, int shape, V3<T> q, V3<T> d, bool out, double lim = kBig) {
   Hit h;
-  each_shape(shape, [&](int u) {
-    by_depth(S, u, [&](auto D) {
-      using C = Csg<T, D(), SC::shape_set, SC::box_on>;
+  each_shape(SC::families_on && S.families, shape, [&](auto one, int u) {
+    by_depth(S, u, one, [&](auto D) {
+      using C = Csg<T, D(), SC::shape_set, SC::box_on, one()>;
       h = out ? C::dist_out(shape_view(S), u, q, d, lim) : C::dist_in(shape_view(S), u, q, d);
     });
   });
@@ -1860,9 +1897,9 @@ __device__ __forceinline__ double shape_polish(const SC& S, int shape, uint32_t 
   const uint32_t path = leaf & 0xffffffu;
   const int depth = int(leaf >> 24);
   double s;
-  each_shape(shape, [&](int u) {
-    by_depth(S, u, [&](auto D) {
-      s = Csg<T, D(), SC::shape_set, SC::box_on>::polish(shape_view(S), u, path, depth, exiting, q, d, s0, back);
+  each_shape(SC::families_on && S.families, shape, [&](auto one, int u) {
+    by_depth(S, u, one, [&](auto D) {
+      s = Csg<T, D(), SC::shape_set, SC::box_on, one()>::polish(shape_view(S), u, path, depth, exiting, q, d, s0, back);
     });
   });
   return s;

@@ -4,8 +4,10 @@
 #pragma once
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstring>
+#include <map>
 #include <string>
 #include <vector>
 
@@ -199,6 +201,33 @@ inline void build_cells(const rb_scene_desc* d, const rb_node_desc& n, std::vect
   }
 }
 
+// Whether kFamilyMin or more of the placed shapes have one structure (see
+// DScene::families). The pairs and triples of alike shapes that most scenes
+// have (two boxes, three aspheric disks) are faster in turns; with up to eight
+// turns before the lanes go together, 85 facets with a shape each take 1.2 to
+// 1.5 times as long.
+constexpr int kFamilyMin = 8;
+inline bool has_families(const std::vector<DShape>& shapes, const std::vector<DNode>& nodes) {
+  std::map<std::array<int, 4>, int> kinds;
+  std::vector<int> kind(shapes.size(), -1);
+  auto kind_of = [&](auto&& self, int i) -> int {
+    int& k = kind[size_t(i)];
+    if (k >= 0) return k;
+    const DShape& s = shapes[size_t(i)];
+    std::array<int, 4> key = {s.type, 0, 0, 0};
+    if (s.type == RB_SHAPE_COMPOSITE) key = {s.type, s.op, self(self, s.left), self(self, s.right)};
+    return k = kinds.emplace(key, int(kinds.size())).first->second;
+  };
+  std::vector<char> placed(shapes.size(), 0);
+  std::vector<int> members(shapes.size(), 0);  // by kind
+  for (const DNode& n : nodes) {
+    if (placed[size_t(n.shape)]) continue;
+    placed[size_t(n.shape)] = 1;
+    if (++members[size_t(kind_of(kind_of, n.shape))] >= kFamilyMin) return true;
+  }
+  return false;
+}
+
 inline bool is_identity(const double* rot) {
   for (int k = 0; k < 9; k++)
     if (rot[k] != (k % 4 == 0 ? 1.0 : 0.0)) return false;
@@ -368,6 +397,7 @@ struct SceneLayout {
   bool has_top_box = false;  // the top node has daughters: their bounding box follows
   float top_lo[3] = {0, 0, 0}, top_hi[3] = {0, 0, 0};
   int32_t top_bvh_lo = 0, top_bvh_n = 0;  // the top node's BVH entries
+  bool families = false;                  // see DScene::families
   int32_t top_leaves = 0;                 // its daughters, the first of the leaves
   int32_t max_depth = 0;                  // deepest boolean nesting of any shape
   bool has_lens = false;                  // a placed node is an ALens
@@ -452,6 +482,7 @@ inline int pack_scene(const rb_scene_desc* d, std::vector<char>& blob, SceneLayo
     if (shapes[i].type == RB_SHAPE_ASPHERIC || shapes[i].type == RB_SHAPE_WINSTON) lay.has_solver = true;
     lay.max_depth = std::max(lay.max_depth, shapes[i].depth);
   }
+  lay.families = has_families(shapes, nodes);
   blob.clear();
   lay.nodes = put(blob, nodes.data(), nodes.size());
   lay.leaves = put(blob, leaves.data(), leaves.size());
@@ -506,6 +537,7 @@ inline DScene scene_view(const char* base, const SceneLayout& lay) {
   s.stage_lo = 0;
   s.stage_n = 0;
   s.leaf_stage_n = 0;
+  s.families = lay.families;
   return s;
 }
 

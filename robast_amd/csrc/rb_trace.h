@@ -139,6 +139,16 @@ __device__ __forceinline__ bool all_one(int n, int& u) {
   u = uniform(n);
   return wave_same(n, u);
 }
+// Runs f(u) for each lane's volume u: with scalar loads where all active lanes
+// name one, else the lanes of the wavefront form (whose sorted rays name few)
+// in turns and those of the others each for itself (a table look-up costs less
+// than a dozen turns).
+template <typename SC, typename F> __device__ __forceinline__ void each_volume(int volume, F&& f) {
+  int u;
+  if constexpr (SC::wave_on) in_turns(volume, f);
+  else if (all_one(volume, u)) f(u);
+  else f(volume);
+}
 // A node's integers
 struct NodeInts {
   int shape, kind, volume, parent, leaf0, n_children, bvh_root;
@@ -902,7 +912,7 @@ __device__ void do_reflection(const SC& S, const TraceParams& P, const IO& io, i
   bool absorbed = false;
   if (kind == RB_KMIRROR) {
     double ref = 1.;
-    each_shape(volume, [&](int u) {
+    each_volume<SC>(volume, [&](int u) {
       const VolumePtr v = (VolumePtr)S.volumes + u;
       ref = v->refl_table >= 0 ? table_eval(S, v->refl_table, L.lambda) : v->refl_const;
     });
@@ -1099,7 +1109,7 @@ __device__ __forceinline__ bool interact(const SC& S, const TraceParams& P, cons
     if (L.npoints == np0) L.p = x1;
   } else if (tn == RB_KFOCUS) {
     double qe = 1.;
-    each_shape(to.volume, [&](int u) {
+    each_volume<SC>(to.volume, [&](int u) {
       const VolumePtr v = (VolumePtr)S.volumes + u;
       if (v->qe_lambda_table >= 0) qe = table_eval(S, v->qe_lambda_table, lambda);
       if (v->qe_angle_table >= 0) qe *= table_eval(S, v->qe_angle_table, cold_acos(dot(L.d, n)));

@@ -81,7 +81,7 @@ __device__ __forceinline__ T prim_dist(int type, ParamPtr p, V3<T> q, V3<T> d, b
   return out ? wave_prim_dist_out<T, SH>(type, (const double*)p, q, d) : wave_prim_dist_in<T, SH>(type, (const double*)p, q, d);
 }
 
-template <typename T, unsigned SH> __device__ __forceinline__ bool flat_contains(const ShapeRef& R, V3<T> q) {
+template <typename T, unsigned SH> __device__ __forceinline__ bool flat_contains(const ShapeRef<>& R, V3<T> q) {
   const bool comp = R.type == RB_SHAPE_COMPOSITE;
   const int op = R.sh->op;
   bool a = false;
@@ -108,7 +108,7 @@ template <typename T, unsigned SH> __device__ __forceinline__ bool flat_contains
 // Distance to enter (out) or leave the shape; see Csg::dist_out / dist_in.
 // A difference's right operand is crossed the other way round.
 template <typename T, unsigned SH>
-__device__ __forceinline__ Hit flat_dist(const ShapeRef& R, bool out, V3<T> q, V3<T> d, double lim) {
+__device__ __forceinline__ Hit flat_dist(const ShapeRef<>& R, bool out, V3<T> q, V3<T> d, double lim) {
   const bool comp = R.type == RB_SHAPE_COMPOSITE;
   const int op = R.sh->op;
   // boundary to boundary: entering an intersection or a difference, leaving a union
@@ -176,7 +176,7 @@ __device__ __forceinline__ Hit flat_dist(const ShapeRef& R, bool out, V3<T> q, V
 }
 
 template <typename T, unsigned SH>
-__device__ __forceinline__ V3<T> flat_normal(const ShapeRef& R, uint32_t leaf, V3<T> q, V3<T> d) {
+__device__ __forceinline__ V3<T> flat_normal(const ShapeRef<>& R, uint32_t leaf, V3<T> q, V3<T> d) {
   const bool comp = R.type == RB_SHAPE_COMPOSITE;
   const int mine = (leaf >> 24) > 0u ? int(leaf & 1u) : 0;
   V3<T> n = mk<T>(T(0), T(0), T(1));
@@ -205,22 +205,22 @@ template <typename T, typename SC>
 __device__ __forceinline__ bool wave_contains(const SC& S, int shape, V3<T> q) {
   static_assert(SC::max_depth == 1, "the wavefront forms handle one nesting level");
   bool in = false;
-  each_shape(shape, [&](int u) { in = flat_contains<T, SC::shape_set>(ShapeRef(shape_view(S), u), q); });
+  in_turns(shape, [&](int u) { in = flat_contains<T, SC::shape_set>(ShapeRef<>(shape_view(S), u), q); });
   return in;
 }
 template <typename T, typename SC>
 __device__ __forceinline__ Hit wave_dist(const SC& S, int shape, V3<T> q, V3<T> d, bool out, double lim) {
   Hit h = {kBig, 0u, 0u};
   // the lanes that enter and those that leave a shape take turns too
-  each_shape(2 * shape + (out ? 1 : 0), [&](int u) {
-    h = flat_dist<T, SC::shape_set>(ShapeRef(shape_view(S), u >> 1), (u & 1) != 0, q, d, lim);
+  in_turns(2 * shape + (out ? 1 : 0), [&](int u) {
+    h = flat_dist<T, SC::shape_set>(ShapeRef<>(shape_view(S), u >> 1), (u & 1) != 0, q, d, lim);
   });
   return h;
 }
 template <typename T, typename SC>
 __device__ __forceinline__ V3<T> wave_normal(const SC& S, int shape, uint32_t leaf, V3<T> q, V3<T> d) {
   V3<T> n = mk<T>(T(0), T(0), T(1));
-  each_shape(shape, [&](int u) { n = flat_normal<T, SC::shape_set>(ShapeRef(shape_view(S), u), leaf, q, d); });
+  in_turns(shape, [&](int u) { n = flat_normal<T, SC::shape_set>(ShapeRef<>(shape_view(S), u), leaf, q, d); });
   return n;
 }
 

@@ -78,9 +78,10 @@ struct rb_scene {
 namespace {
 
 // The scene as the kernels compiled for composites at most MAXD deep take it.
-template <int MAXD, bool BORDERS = false, bool BOX = false, bool LENS = true, bool SOLVER = true, bool WAVE = false>
-DSceneOf<MAXD, BORDERS, (MAXD > 1), BOX, LENS, SOLVER, WAVE> scene_of(const rb_scene* sc) {
-  DSceneOf<MAXD, BORDERS, (MAXD > 1), BOX, LENS, SOLVER, WAVE> s;
+template <int MAXD, bool BORDERS = false, bool BOX = false, bool LENS = true, bool SOLVER = true, bool WAVE = false,
+          bool FAM = (MAXD == 1 && !BOX)>
+DSceneOf<MAXD, BORDERS, (MAXD > 1), BOX, LENS, SOLVER, WAVE, FAM> scene_of(const rb_scene* sc) {
+  DSceneOf<MAXD, BORDERS, (MAXD > 1), BOX, LENS, SOLVER, WAVE, FAM> s;
   static_cast<DScene&>(s) = sc->s;
   return s;
 }
@@ -436,8 +437,8 @@ __global__ void __launch_bounds__(256) k_unstage(const RayRec* rr, RayIO io, int
 // input order). A ray is traced from start to end by the lane that claimed
 // it, with the same per-ray Philox stream, so results equal k_trace's. Every
 // wave leaves when the counter has passed n and none of its lanes holds a ray.
-template <bool MIXED, int MAXD, bool BORDERS>
-__global__ void __launch_bounds__(kTraceBlock) RB_TRACE_ATTR k_trace_persist(DSceneOf<MAXD, BORDERS, (MAXD > 1), true> S, RayIO io,
+template <bool MIXED, int MAXD, bool BORDERS, bool FAM>
+__global__ void __launch_bounds__(kTraceBlock) RB_TRACE_ATTR k_trace_persist(DSceneOf<MAXD, BORDERS, (MAXD > 1), true, true, true, false, FAM> S, RayIO io,
                                                                           int64_t n,
                                                                           TraceParams P,
                                                                           unsigned long long* next_ray,
@@ -530,8 +531,8 @@ struct PoolLDS {
   int32_t taken[kPoolBlock];
 };
 
-template <bool MIXED, int MAXD, bool BORDERS>
-__global__ void __launch_bounds__(kPoolBlock) RB_TRACE_ATTR k_trace_regroup(DSceneOf<MAXD, BORDERS, (MAXD > 1), true> S, RayIO io,
+template <bool MIXED, int MAXD, bool BORDERS, bool FAM>
+__global__ void __launch_bounds__(kPoolBlock) RB_TRACE_ATTR k_trace_regroup(DSceneOf<MAXD, BORDERS, (MAXD > 1), true, true, true, false, FAM> S, RayIO io,
                                                                           int64_t n, TraceParams P,
                                                                           unsigned long long* next_ray,
                                                                           const uint32_t* perm, RayRec* rr) {
@@ -660,9 +661,9 @@ template <typename SC> struct TraceArgs {
   const uint32_t* perm;
   RayRec* rr;
 };
-template <bool MIXED, int MAXD, bool BORDERS, bool LENS, bool SOLVER, bool WAVE>
+template <bool MIXED, int MAXD, bool BORDERS, bool LENS, bool SOLVER, bool WAVE, bool FAM>
 __global__ void __launch_bounds__(kTraceBlock) RB_WAVE_ATTR(WAVE)
-    k_trace(TraceArgs<DSceneOf<MAXD, BORDERS, (MAXD > 1), false, LENS, SOLVER, WAVE>> A) {
+    k_trace(TraceArgs<DSceneOf<MAXD, BORDERS, (MAXD > 1), false, LENS, SOLVER, WAVE, FAM>> A) {
   __shared__ int32_t cand_node[kCand * kCandStride];
   __shared__ float cand_tn[kCand * kCandStride];
   const auto& S = A.S;
@@ -684,7 +685,7 @@ __global__ void __launch_bounds__(kTraceBlock) RB_WAVE_ATTR(WAVE)
   L.cand = {cand_node + threadIdx.x, cand_tn + threadIdx.x};
   L.ray = P.id_base + uint64_t(i);
   NoRecord rec;
-  const KernelRays<TraceArgs<DSceneOf<MAXD, BORDERS, (MAXD > 1), false, LENS, SOLVER, WAVE>>> io{
+  const KernelRays<TraceArgs<DSceneOf<MAXD, BORDERS, (MAXD > 1), false, LENS, SOLVER, WAVE, FAM>>> io{
       A.io.path_cap, (const char*)__builtin_amdgcn_kernarg_segment_ptr()};
   trace_lane<MIXED>(S, P, io, i, L, rec, act, &i);
   if (!act) return;
@@ -704,7 +705,7 @@ __global__ void __launch_bounds__(kTraceBlock) RB_WAVE_ATTR(WAVE)
 constexpr int kAdjWaveAcc = 800;  // entries of one group's sums
 template <bool MIXED, int MAXD, bool LENS = true, bool SOLVER = true, bool WAVE = false>
 __global__ void __launch_bounds__(kTraceBlock) RB_WAVE_ATTR(WAVE)
-    k_adjoint(DSceneOf<MAXD, false, (MAXD > 1), false, LENS, SOLVER, WAVE> S, RayIO io, int64_t n, TraceParams P, AdjParams A,
+    k_adjoint(DSceneOf<MAXD, false, (MAXD > 1), false, LENS, SOLVER, WAVE, true> S, RayIO io, int64_t n, TraceParams P, AdjParams A,
               double* grad, const uint32_t* perm, const RayRec* rr) {
   __shared__ double acc[WAVE ? kAdjWaveAcc : kMaxAdjAcc];
   const int block = adj_block(A.mode, A.n_params);
@@ -1179,43 +1180,62 @@ static TraceArgs<SC> trace_args(const SC& S, const RayIO& io, int64_t n, const T
 constexpr int64_t kSmallBatchRays = int64_t(1) << 15;
 constexpr int kSmallTraceBlock = 64;
 
-template <bool MIXED, int MAXD, bool BORDERS, bool LENS, bool SOLVER, bool WAVE>
+template <bool MIXED, int MAXD, bool BORDERS, bool LENS, bool SOLVER, bool WAVE, bool FAM = (MAXD == 1)>
 static void launch_lane(rb_ctx* ctx, const rb_scene* scene, const RayIO& io, int64_t n, const TraceParams& P,
                         const uint32_t* perm, RayRec* rr) {
   const int block = !perm && n <= kSmallBatchRays ? kSmallTraceBlock : kTraceBlock;
-  hipLaunchKernelGGL((k_trace<MIXED, MAXD, BORDERS, LENS, SOLVER, WAVE>), dim3(unsigned((n + block - 1) / block)),
+  hipLaunchKernelGGL((k_trace<MIXED, MAXD, BORDERS, LENS, SOLVER, WAVE, FAM>), dim3(unsigned((n + block - 1) / block)),
                      dim3(block), 0, ctx->stream,
-                     trace_args(scene_of<MAXD, BORDERS, false, LENS, SOLVER, WAVE>(scene), io, n, P, perm, rr));
+                     trace_args(scene_of<MAXD, BORDERS, false, LENS, SOLVER, WAVE, FAM>(scene), io, n, P, perm, rr));
+}
+
+// A work-queue kernel (PERSISTENT or REGROUP).
+template <bool MIXED, int MAXD, bool BORDERS, bool FAM>
+static int launch_queue(rb_ctx* ctx, const rb_scene* scene, bool regroup, const RayIO& io, int64_t n,
+                        const TraceParams& P, const uint32_t* perm, RayRec* rr, unsigned long long* counter,
+                        bool clear_by_kernel) {
+  const void* fn = regroup ? (const void*)k_trace_regroup<MIXED, MAXD, BORDERS, FAM>
+                           : (const void*)k_trace_persist<MIXED, MAXD, BORDERS, FAM>;
+  const int pblock = regroup ? kPoolBlock : kTraceBlock;
+  int per_cu = 0;
+  HIPCHK(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, pblock, 0));
+  // (the regrouping form's wavefronts take 64 rays each from the start, so a
+  // small batch is spread over the machine)
+  const int64_t pgrid = std::min<int64_t>((n + (regroup ? 64 : pblock) - 1) / (regroup ? 64 : pblock),
+                                          int64_t(std::max(per_cu, 1)) * ctx->cus);
+  if (clear_by_kernel)
+    hipLaunchKernelGGL(k_clear_counter, dim3(1), dim3(64), 0, ctx->stream, counter);
+  else
+    HIPCHK(ctx, hipMemsetAsync(counter, 0, sizeof(unsigned long long), ctx->stream));
+  const auto S = scene_of<MAXD, BORDERS, true, true, true, false, FAM>(scene);
+  if (regroup)
+    hipLaunchKernelGGL((k_trace_regroup<MIXED, MAXD, BORDERS, FAM>), dim3(unsigned(pgrid)), dim3(pblock), 0,
+                       ctx->stream, S, io, n, P, counter, perm, rr);
+  else
+    hipLaunchKernelGGL((k_trace_persist<MIXED, MAXD, BORDERS, FAM>), dim3(unsigned(pgrid)), dim3(pblock), 0,
+                       ctx->stream, S, io, n, P, counter, perm, rr);
+  return 0;
 }
 
 // The trace kernel for the scene's depth and the lane schedule. Rays in
 // coherence order, in scenes whose composites nest one level, without a
-// refracting volume, are navigated a wavefront at a time.
+// refracting volume, are navigated a wavefront at a time. The work-queue and
+// the deep lane kernels for scenes with families (FAM) are compiled once, with
+// everything else in.
 template <bool MIXED, int MAXD, bool BORDERS>
 static int launch_trace(rb_ctx* ctx, const rb_scene* scene, int schedule, const RayIO& io, int64_t n,
                         const TraceParams& P, const uint32_t* perm, RayRec* rr, unsigned long long* counter,
                         bool clear_by_kernel) {
+  const bool families = scene->s.families;
   if (schedule != RB_SCHEDULE_LANE) {
     const bool regroup = schedule == RB_SCHEDULE_REGROUP;
-    const void* fn = regroup ? (const void*)k_trace_regroup<MIXED, MAXD, BORDERS>
-                             : (const void*)k_trace_persist<MIXED, MAXD, BORDERS>;
-    const int pblock = regroup ? kPoolBlock : kTraceBlock;
-    int per_cu = 0;
-    HIPCHK(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, pblock, 0));
-    // (the regrouping form's wavefronts take 64 rays each from the start, so a
-    // small batch is spread over the machine)
-    const int64_t pgrid = std::min<int64_t>((n + (regroup ? 64 : pblock) - 1) / (regroup ? 64 : pblock),
-                                            int64_t(std::max(per_cu, 1)) * ctx->cus);
-    if (clear_by_kernel)
-      hipLaunchKernelGGL(k_clear_counter, dim3(1), dim3(64), 0, ctx->stream, counter);
-    else
-      HIPCHK(ctx, hipMemsetAsync(counter, 0, sizeof(unsigned long long), ctx->stream));
-    if (regroup)
-      hipLaunchKernelGGL((k_trace_regroup<MIXED, MAXD, BORDERS>), dim3(unsigned(pgrid)), dim3(pblock), 0, ctx->stream,
-                         scene_of<MAXD, BORDERS, true>(scene), io, n, P, counter, perm, rr);
-    else
-      hipLaunchKernelGGL((k_trace_persist<MIXED, MAXD, BORDERS>), dim3(unsigned(pgrid)), dim3(pblock), 0, ctx->stream,
-                         scene_of<MAXD, BORDERS, true>(scene), io, n, P, counter, perm, rr);
+    const int rc = families ? launch_queue<MIXED, MAXD, true, true>(ctx, scene, regroup, io, n, P, perm, rr, counter,
+                                                                    clear_by_kernel)
+                            : launch_queue<MIXED, MAXD, BORDERS, false>(ctx, scene, regroup, io, n, P, perm, rr,
+                                                                        counter, clear_by_kernel);
+    if (rc) return rc;
+  } else if (MAXD > 1 && families) {
+    launch_lane<MIXED, MAXD, true, true, true, false, true>(ctx, scene, io, n, P, perm, rr);
   } else if (scene->has_lens) {
     launch_lane<MIXED, MAXD, BORDERS, true, true, false>(ctx, scene, io, n, P, perm, rr);
   } else if (scene->has_solver) {
@@ -2140,7 +2160,7 @@ int rbgpu_adjoint(rb_ctx* ctx, const rb_scene* scene, const rb_trace_opts* opts,
                        n, P, A, grad, perm, rr);
   else if (opts->precision == RB_PRECISION_MIXED)
     hipLaunchKernelGGL((k_adjoint<true, kMaxCsgDepth>), dim3(unsigned(grid)), dim3(block), 0, ctx->stream,
-                       scene_of<kMaxCsgDepth>(scene), io, n, P, A, grad, perm, rr);
+                       scene_of<kMaxCsgDepth, false, false, true, true, false, true>(scene), io, n, P, A, grad, perm, rr);
   else if (wave && !scene->has_solver)  // sorted: a wavefront at a time
     hipLaunchKernelGGL((k_adjoint<false, 1, false, false, true>), dim3(unsigned(grid)), dim3(block), 0, ctx->stream, scene_of<1, false, false, false, false, true>(scene), io, n,
                        P, A, grad, perm, rr);
@@ -2158,10 +2178,10 @@ int rbgpu_adjoint(rb_ctx* ctx, const rb_scene* scene, const rb_trace_opts* opts,
                        io, n, P, A, grad, perm, rr);
   else if (!scene->has_lens)
     hipLaunchKernelGGL((k_adjoint<false, kMaxCsgDepth, false>), dim3(unsigned(grid)), dim3(block), 0, ctx->stream,
-                       scene_of<kMaxCsgDepth, false, false, false>(scene), io, n, P, A, grad, perm, rr);
+                       scene_of<kMaxCsgDepth, false, false, false, true, false, true>(scene), io, n, P, A, grad, perm, rr);
   else
     hipLaunchKernelGGL((k_adjoint<false, kMaxCsgDepth>), dim3(unsigned(grid)), dim3(block), 0, ctx->stream,
-                       scene_of<kMaxCsgDepth>(scene), io, n, P, A, grad, perm, rr);
+                       scene_of<kMaxCsgDepth, false, false, true, true, false, true>(scene), io, n, P, A, grad, perm, rr);
   HIPCHK(ctx, hipGetLastError());
   HIPCHK(ctx, hipEventRecord(ctx->evk1, ctx->stream));
   HIPCHK(ctx, hipEventRecord(ctx->ev1, ctx->stream));
