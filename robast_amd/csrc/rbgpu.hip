@@ -1360,14 +1360,15 @@ static int launch_order_key(rb_ctx* ctx, const rb_scene* scene, const RayIO& io,
 // 30-bit keys take 3 passes instead of 4 (blocks of 1024 threads x 8 keys).
 // Measured on the 1e7-ray Davies-Cotton, whole trace: 6.15 ms with rocPRIM's
 // default (8 bits), 6.02 with this; 10 bits on 512 x 12, 512 x 24 or
-// 1024 x 4 gained nothing, 11 bits lost 0.25 ms. Up to 2^18 pairs are merge
-// sorted (2e5: 0.110 ms for the whole ordering, 0.116 by onesweep; rocPRIM's
-// limit of 2^20 cost 0.06-0.08 ms from 3e5 to 9e5: 0.178 -> 0.125, 0.270 -> 0.192).
+// 1024 x 4 gained nothing, 11 bits lost 0.25 ms. Up to 2^16 pairs are merge
+// sorted (whole sorted trace, Davies-Cotton, us: 4e4 rays 177 merged and 180 by
+// onesweep's two passes, 6.6e4 189 and 182, 1.3e5 207 and 201, 2.25e5 275 and
+// 232, 2.62e5 313 and 265).
 using OrderSortConfig = rocprim::radix_sort_config<
     rocprim::default_config, rocprim::default_config,
     rocprim::radix_sort_onesweep_config<rocprim::kernel_config<1024, 8>, rocprim::kernel_config<1024, 8>, 10,
                                         rocprim::block_radix_rank_algorithm::match>,
-    262144>;
+    65536>;
 
 // Coherence order of n rays: keys from k_order_key, then a radix sort of
 // (key, index) pairs. *perm receives the sorted indices (device). With rr,
