@@ -228,8 +228,10 @@ typedef struct {
  * ray, grown on demand), read and written by the trace and copied back to
  * the ray arrays after it. AUTO sorts batches of 2^20 rays or more; of 2^18 or
  * more when the work-queue schedule traces them or the top volume has at
- * least 16 daughters; of 3 x 2^16 or more in scenes with aspheric disks or
- * Winston cones traced one lane per ray. */
+ * least 16 daughters (FP64 gradients of such scenes: of 5 x 2^16 or more); of
+ * 3 x 2^16 or more in scenes with aspheric disks or Winston cones traced one
+ * lane per ray. It cannot see whether the input is coherent as given, as a grid
+ * of parallel rays is: up to about 2^19 of those are faster with INPUT. */
 enum { RB_ORDER_AUTO = 0, RB_ORDER_INPUT = 1, RB_ORDER_COHERENT = 2 };
 
 /* Lane schedule. LANE: one lane per ray for the whole trace. PERSISTENT: a

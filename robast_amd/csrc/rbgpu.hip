@@ -1290,19 +1290,30 @@ constexpr int64_t kAutoOrderMin = int64_t(1) << 20;
 constexpr int64_t kAutoOrderMinQueue = int64_t(1) << 18;
 
 // Lane-schedule scenes whose rays cost more than a few boxes gain from the
-// order earlier, as the sorted rays are navigated a wavefront at a time (whole
-// trace, input order against sorted, ms): with iterative solvers from 3 x 2^16
-// rays on (Schwarzschild-Couder 1e5 0.35 and 0.40, 2e5 0.66 and 0.48, 5e5 1.1
-// and 0.79), with many daughters in the top node from 2^18 on (Davies-Cotton
-// 1e5 0.16 and 0.21, 2e5 0.28 and 0.24, 5e5 0.55 and 0.40; a shower's photons,
-// of which several share a path, 2.2e5 0.24 and 0.29).
+// order earlier (whole trace, input order against sorted, us; the wavefront
+// form navigates sorted FP64 rays in scenes one level deep): with iterative
+// solvers from 3 x 2^16 rays on (Schwarzschild-Couder 2.25e5 644 and 470, 3e5
+// 822 and 562), with many daughters in the top node from 2^18 on (Davies-Cotton
+// 2.63e5 387 and 268, 6e5 693 and 397; a shower's photons, of which several
+// share a path, 2.63e5 315 and 269, but 1.97e5 240 and 232). Random rays gain
+// without that form too (at 2.63e5 and 6e5: mixed 413 and 328, 730 and 517; two
+// levels deep 654 and 455, 1179 and 788; mixed gradient 516 and 365, 914 and
+// 623; the allocation-free trace 404 and 371, 693 and 534 at 3e5 and 6e5). A
+// grid of parallel rays loses here as above, up to there (2.63e5 and 6e5: FP64
+// 204 and 215, 373 and 342; mixed 219 and 293, 423 and 434; two levels deep 354
+// and 416, 667 and 664; aspheric 332 and 361, 635 and 600).
 constexpr int64_t kAutoOrderMinSolver = int64_t(3) << 16;
 constexpr int64_t kAutoOrderMinDaughters = int64_t(1) << 18;
 constexpr int kManyDaughters = 16;
-static int64_t auto_order_min(const rb_scene* scene, bool queue) {
+// The wavefront form's gradient of many facets, whose rays are sorted within
+// their groups, gains later (8 groups, us: 2.63e5 rays 450 and 481, 3e5 465 and
+// 484, 3.5e5 493 and 485, 4e5 608 and 518).
+constexpr int64_t kAutoOrderMinFacetGradient = int64_t(5) << 16;
+static int64_t auto_order_min(const rb_scene* scene, bool queue, bool wave_gradient = false) {
   if (queue) return kAutoOrderMinQueue;
   if (scene->has_solver) return kAutoOrderMinSolver;
-  return scene->top_daughters >= kManyDaughters ? kAutoOrderMinDaughters : kAutoOrderMin;
+  if (scene->top_daughters < kManyDaughters) return kAutoOrderMin;
+  return wave_gradient ? kAutoOrderMinFacetGradient : kAutoOrderMinDaughters;
 }
 
 // Sort bits of the coherence order of n rays: the tile index in the high
@@ -2140,15 +2151,15 @@ int rbgpu_adjoint(rb_ctx* ctx, const rb_scene* scene, const rb_trace_opts* opts,
   A.weight = adj->weight;
   const int block = kTraceBlock;
   const int64_t grid = (n + block - 1) / block;
-  const bool coherent = scene->has_top_box && n < (int64_t(1) << 31) &&
-                        (opts->order == RB_ORDER_COHERENT ||
-                         (opts->order == RB_ORDER_AUTO && n >= auto_order_min(scene, false)));
-  const uint32_t* perm = nullptr;
-  RayRec* rr = nullptr;
   const bool shallow = scene->max_depth <= 1 && !scene->has_ext;
   // the wavefront form: one group's sums in LDS, the rays ordered by group
   const bool wave_fits = shallow && !scene->has_lens && opts->precision != RB_PRECISION_MIXED &&
                          adj_block(adj->mode, adj->n_params) <= kAdjWaveAcc;
+  const bool coherent = scene->has_top_box && n < (int64_t(1) << 31) &&
+                        (opts->order == RB_ORDER_COHERENT ||
+                         (opts->order == RB_ORDER_AUTO && n >= auto_order_min(scene, false, wave_fits)));
+  const uint32_t* perm = nullptr;
+  RayRec* rr = nullptr;
   HIPCHK(ctx, hipEventRecord(ctx->ev0, ctx->stream));
   if (coherent) {
     const int rc = order_rays(ctx, scene, io, n, &perm, &rr, false, wave_fits ? group_size : 0, groups);
