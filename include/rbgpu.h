@@ -276,7 +276,13 @@ typedef struct rb_ctx rb_ctx;
 typedef struct rb_scene rb_scene;
 
 /* Create a context on HIP device `device` with its own stream (default
- * priority). Contexts are not to be shared across host threads. */
+ * priority). Contexts are not to be shared across host threads.
+ * A context keeps memory from call to call, grown on demand, until it is
+ * destroyed: device memory for the arrays of a host batch, of photon bunches
+ * or of a histogram (as large as the largest such call so far, up to 1 GiB;
+ * larger calls allocate their own), pinned host memory for host batches of up
+ * to 16 MiB (16 MiB at most), and 16 + 128 B per ray of its largest sorted
+ * batch. */
 int rbgpu_ctx_create(int device, rb_ctx** out);
 void rbgpu_ctx_destroy(rb_ctx* ctx);
 const char* rbgpu_last_error(const rb_ctx* ctx);

@@ -141,7 +141,7 @@ struct DSceneOf : DScene {
 };
 
 // Shape records and parameters are read through the constant address space:
-// the shape code runs with one shape for the whole wavefront (each_shape),
+// the shape code mostly runs with one shape for the whole wavefront (each_shape),
 // so the address is uniform and the compiler reads them with scalar loads
 // into scalar registers -- no vector load latency, no vector registers and
 // no per-lane address arithmetic. (Where a lane reads a shape of its own the

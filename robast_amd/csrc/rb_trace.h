@@ -10,9 +10,11 @@ inline long rb_emul_fallbacks = 0;
 // host views are never staged (stage_n = 0)
 inline DBvh bvh_node(const DScene& S, int i) { return S.bvh[i]; }
 #else
-// LDS copies of the top node's BVH (DScene::stage_lo / stage_n) and of its
-// daughters' boxes (DScene::leaf_stage_n), written by stage_bvh() at the entry
-// of every kernel that navigates.
+// LDS copies of the top node's BVH (DScene::stage_lo / stage_n), written by
+// stage_bvh() at the entry of the kernels that navigate lane by lane, and of its
+// daughters' boxes (DScene::leaf_stage_n), written by stage_leaves() at the entry
+// of those that navigate a wavefront at a time. bvh_node() is for the former
+// only: the others leave its copy unwritten.
 __shared__ __attribute__((aligned(16))) DBvh g_bvh_stage[kBvhStage];  // read as float4 pairs
 __shared__ __attribute__((aligned(16))) DBvh g_leaf_stage[kLeafStage];
 
@@ -152,19 +154,17 @@ template <typename SC, typename F> __device__ __forceinline__ void each_volume(i
 // A node's integers
 struct NodeInts {
   int shape, kind, volume, parent, leaf0, n_children, bvh_root;
-  bool turned;
 };
 __device__ __forceinline__ NodeInts node_ints(const DScene& S, int n) {
   NodeInts r;
   int u;
   if (all_one(n, u)) {
     const NodePtr a = node_ptr(S, u);
-    r = {a->shape, a->kind, a->volume, a->parent, a->leaf0, a->n_children, a->bvh_root, false};
+    r = {a->shape, a->kind, a->volume, a->parent, a->leaf0, a->n_children, a->bvh_root};
   } else {
     const DNode* a = S.nodes + n;
-    r = {a->shape, a->kind, a->volume, a->parent, a->leaf0, a->n_children, a->bvh_root, false};
+    r = {a->shape, a->kind, a->volume, a->parent, a->leaf0, a->n_children, a->bvh_root};
   }
-  r.turned = (r.kind & kNodeTurned) != 0;
   r.kind &= ~kNodeTurned;
   return r;
 }
@@ -200,6 +200,7 @@ __device__ __forceinline__ DBvh cell_at(const SC& S, int n, int hint, float fx, 
 // tested instead of the walk: the same candidates, the same answer.
 template <typename SC>
 __device__ int first_daughter_containing(const SC& S, int n, V3<double> p, int skip, int hint = -1) {
+  static_assert(!SC::wave_on, "reads the staged BVH");
   const DNode& nd = S.nodes[n];
   if (nd.n_children == 0) return -1;
   const float fx = float(p.x), fy = float(p.y), fz = float(p.z);
@@ -625,6 +626,7 @@ __device__ bool search_boundary_mixed(const SC& S, int cur, V3<double> p, V3<dou
 // whose rays bounce many times inside light guides, compile it in).
 template <bool MIXED, bool HINT = false, typename SC>
 __device__ int next_boundary(const SC& S, Lane& L) {
+  static_assert(!SC::wave_on, "reads the staged BVH");
   double extra = L.on_b ? kTol : 0.0;
   L.on_b = false;
   L.p = axpy(L.p, extra, L.d);

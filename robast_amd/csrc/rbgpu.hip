@@ -346,10 +346,10 @@ __device__ __forceinline__ uint32_t spread3(uint32_t v) {
 constexpr int kOrderTileBits = RB_ORDER_TILE_BITS;
 constexpr int kOrderGlobalBits = 31;  // one tile: batches are below 2^31 rays
 // Keys are 32-bit: the tile index in the high bits and as many of the top
-// bits of the 30-bit Morton code as fit below it (all 30 for a global order
-// or up to 4 tiles; 27 = 9 bits per axis for 2^19-ray tiles at 1e7 rays),
-// so that the radix sort moves 8-byte pairs (3 passes of 10 bits for the
-// global order, 4 of 8 in the allocation-free entry point) instead of
+// bits of the 30-bit Morton code as fit below it (from kShortKeyRays on all 30
+// for a global order or up to 4 tiles, below it 20; see key_bits), so that the
+// radix sort moves 8-byte pairs (3 or 2 passes of 10 bits for the global order,
+// 4 or 3 of 8 in the allocation-free entry point) instead of
 // 12-byte ones. The walk reads the top node's BVH through the same LDS copy
 // as the tracing kernels (stage_bvh / bvh_node): it is a chain of dependent
 // loads, and LDS answers them at a fraction of the L2 latency.
@@ -702,7 +702,10 @@ __global__ void __launch_bounds__(kTraceBlock) RB_WAVE_ATTR(WAVE)
 // then holds one group's rays, rarely two, and needs that group's sums in LDS
 // only (a ray of another group adds to the result itself), which leaves room
 // for three wavefronts per SIMD.
-constexpr int kAdjWaveAcc = 800;  // entries of one group's sums
+// (Entries of one group's sums: enough for 88 facets, 3 x 265 + 4. With the
+// form's other 43 KB three blocks share the 160 KB of LDS up to about 1,400;
+// larger groups than 800 have not been timed and stay with the lane form.)
+constexpr int kAdjWaveAcc = 800;
 template <bool MIXED, int MAXD, bool LENS = true, bool SOLVER = true, bool WAVE = false>
 __global__ void __launch_bounds__(kTraceBlock) RB_WAVE_ATTR(WAVE)
     k_adjoint(DSceneOf<MAXD, false, (MAXD > 1), false, LENS, SOLVER, WAVE, true> S, RayIO io, int64_t n, TraceParams P, AdjParams A,
@@ -1317,7 +1320,7 @@ static int64_t auto_order_min(const rb_scene* scene, bool queue, bool wave_gradi
 }
 
 // Sort bits of the coherence order of n rays: the tile index in the high
-// bits, as many Morton bits below it as fit in 32.
+// bits, up to key_bits(n) Morton bits below it, as many as fit in 32.
 struct OrderBits {
   int tile_bits;  // rays per tile: 2^tile_bits
   int mbits;
